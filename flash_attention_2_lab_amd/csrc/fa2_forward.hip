@@ -642,7 +642,9 @@ void fa2_forward_d64_kernel(const _Float16* __restrict__ query,
 // then buffer_load_dwordx4 ... lds. The compiler does not track these loads, so it
 // adds no waits for them; the kernel waits with explicit vmcnt. M0 is a reserved
 // register that the compiler sets before each of its own uses, so listing it as
-// clobbered is only documentation (clang warns about reserved clobbers).
+// clobbered is only documentation (clang warns about reserved clobbers). An LDS-DMA needs
+// one wait state after a scalar write of M0, which the compiler inserts for the builtin
+// and not inside inline assembly: the s_nop.
 //  - dma16_asm: tile offset in the scalar offset, for tiles inside the slab.
 //  - dma16_asm_checked: the whole byte offset in the VGPR offset, which the buffer
 //    unit checks against num_records (the scalar offset is not checked), so rows at
@@ -651,13 +653,13 @@ void fa2_forward_d64_kernel(const _Float16* __restrict__ query,
 #pragma clang diagnostic ignored "-Winline-asm"
 __device__ __forceinline__ void dma16_asm(u32x4 src, uint32_t lds_addr, int lane_offset,
                                           int src_offset) {
-    asm volatile("s_mov_b32 m0, %0\n\tbuffer_load_dwordx4 %1, %2, %3 offen lds"
+    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tbuffer_load_dwordx4 %1, %2, %3 offen lds"
                  :: "s"(__builtin_amdgcn_readfirstlane(lds_addr)), "v"(lane_offset), "s"(src),
                     "s"(__builtin_amdgcn_readfirstlane(src_offset))
                  : "memory", "m0");
 }
 __device__ __forceinline__ void dma16_asm_checked(u32x4 src, uint32_t lds_addr, int offset) {
-    asm volatile("s_mov_b32 m0, %0\n\tbuffer_load_dwordx4 %1, %2, 0 offen lds"
+    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tbuffer_load_dwordx4 %1, %2, 0 offen lds"
                  :: "s"(__builtin_amdgcn_readfirstlane(lds_addr)), "v"(offset), "s"(src)
                  : "memory", "m0");
 }
