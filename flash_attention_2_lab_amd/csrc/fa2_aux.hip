@@ -147,7 +147,9 @@ __global__ __launch_bounds__(256) void scores_f32_kernel(const float* __restrict
         else fetch_unit(wave < 2 ? key : query, (wave < 2 ? col * kScoreTile : row0) + 32 * (wave & 1), chunk,
                         lds + wave * kUnitBytes, 0);
     };
-    auto landed = [&]() { asm volatile("s_waitcnt vmcnt(0)\n\ts_barrier" ::: "memory"); };
+    // The wave's fetches have landed and its LDS reads are done: behind the barrier the other
+    // waves read the one slot and refill the other.
+    auto landed = [&]() { asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)\n\ts_barrier" ::: "memory"); };
 
     const uint32_t lane_read = smem_addr + (uint32_t)(m * 256 + ((h ^ (m & 15)) << 4));
     auto read = [&](int slot, int unit, int j) {
@@ -220,7 +222,7 @@ __global__ __launch_bounds__(256) void scores_f32_kernel(const float* __restrict
         for (int i = 0; i < 16; ++i)
             __builtin_amdgcn_raw_buffer_store_b32(__float_as_uint((acc[0][i] + acc[1][i]) * scale), out,
                                                   lane_offset + (8 * (i >> 2) + (i & 3)) * seq_len * 4, 0, 0);
-        asm volatile("s_barrier" ::: "memory");
+        asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
     }
 }
 

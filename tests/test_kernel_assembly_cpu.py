@@ -98,3 +98,16 @@ def test_lds_dma_waits_for_m0_and_its_scalar_operands(kernels):
             gap = _states_since(body, at, lambda past: past.startswith("v_") and bool(_written(past) & read), 5)
             assert gap >= 5, f"{name}: {gap} wait states before {instruction}"
     assert fetches > 1000  # every LDS-DMA kernel was read
+
+
+def test_scores_barriers_wait_for_lds_reads(kernels):
+    """Behind each barrier of the scores kernel another wave's LDS-DMA refills the ring slot that
+    this wave read before it, so the wave waits for its reads at the barrier itself."""
+    scores = {name: body for name, body in kernels.items() if "scores_f32_kernel" in name}
+    assert len(scores) == 4
+    for name, body in scores.items():
+        barriers = [at for at, instruction in enumerate(body) if instruction == "s_barrier"]
+        assert barriers
+        for at in barriers:
+            wait = body[at - 1]
+            assert wait.startswith("s_waitcnt") and "lgkmcnt(0)" in wait, f"{name}: {wait}"
