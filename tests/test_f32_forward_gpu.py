@@ -100,6 +100,32 @@ def test_f32_forward_keeps_small_and_large_values(batch_heads, dim, exponent):
     assert ((out - expected).abs() <= ATOL * scale).all()
 
 
+# Scores of 2^40 and more, whose product with log2(e) rounds by more than a float's exponents
+# span: each row is its largest score's value row. The scores' own errors, 2^-20 of them at most,
+# stay far below the gaps between them.
+@pytest.mark.parametrize("dim", [64, 128])
+@pytest.mark.parametrize("batch_heads", HEADS)
+def test_f32_forward_huge_scores(batch_heads, dim):
+    q, k, v = _inputs(batch_heads, 197, dim, seed=8)
+    q[0, 0] *= 2.0 ** 20
+    k[0, 0] *= 2.0 ** 20
+    # Growing along the keys, so that the running max passes from ordinary to huge values.
+    k[0, -1] *= torch.logspace(0, 50, 197, base=2.0, device="cuda").unsqueeze(-1)
+    out = capi.attention_forward_f32(q, k, v).double().cpu()
+    torch.testing.assert_close(out, _exact(q, k, v), atol=ATOL, rtol=0)
+
+
+@pytest.mark.parametrize("batch_heads", HEADS)
+def test_f32_forward_huge_negative_scores(batch_heads):
+    """Every score of every row below -2^38, from one product each: the smallest one wins."""
+    q, k, v = _inputs(batch_heads, 197, 64, seed=9)
+    q[..., 1:], k[..., 1:] = 0.0, 0.0
+    q[..., 0] = (q[..., 0].abs() + 1.0) * 2.0 ** 20
+    k[..., 0] = -(k[..., 0].abs() + 1.0) * 2.0 ** 21
+    out = capi.attention_forward_f32(q, k, v).double().cpu()
+    torch.testing.assert_close(out, _exact(q, k, v), atol=ATOL, rtol=0)
+
+
 # Scores: 64 x 64 blocks of 32 x 32, dimensions in chunks of 64; 4-byte fetches when the
 # head dimension is not a multiple of 4 or the storage is 4-byte aligned.
 @pytest.mark.parametrize("offset", [0, 1])
