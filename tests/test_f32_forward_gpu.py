@@ -126,6 +126,33 @@ def test_f32_forward_huge_negative_scores(batch_heads):
     torch.testing.assert_close(out, _exact(q, k, v), atol=ATOL, rtol=0)
 
 
+# A score of one product is exact, so a probability of 2^-122 is off by the rounding of its
+# exponent, 122 * 2^-24, and what exp2 and the sums add: 1.5e-5 in all.
+@pytest.mark.parametrize("case", ["zero_value", "large_values", "small_value"])
+@pytest.mark.parametrize("batch_heads", HEADS)
+def test_f32_forward_keeps_small_weights(batch_heads, case):
+    """What a probability near the smallest float, or a value below it, gives keeps its bits
+    when it is what the result consists of."""
+    q, k, v = _inputs(batch_heads, 197, 64, seed=10)
+    gen = torch.Generator().manual_seed(11)
+    low, high = (-200.0, -190.0) if case == "small_value" else (-85.0, -83.0)
+    q.zero_()
+    k.zero_()
+    q[..., 0] = 8.0
+    k[..., 0] = (low + (high - low) * torch.rand(batch_heads, 197, generator=gen)).cuda()
+    k[..., 100, 0] = 0.0  # every row sees key 100 with probability 1
+    v = v.abs() + 0.5
+    if case == "zero_value":
+        v[..., 100, :] = 0.0
+    elif case == "large_values":
+        v *= 2.0 ** 122
+        v[..., 100, :] *= 2.0 ** -122
+    else:
+        v[..., 100, :] *= 2.0 ** -121
+    out = capi.attention_forward_f32(q, k, v).double().cpu()
+    torch.testing.assert_close(out, _exact(q, k, v), atol=0, rtol=2e-5)
+
+
 # Scores: 64 x 64 blocks of 32 x 32, dimensions in chunks of 64; 4-byte fetches when the
 # head dimension is not a multiple of 4 or the storage is 4-byte aligned.
 @pytest.mark.parametrize("offset", [0, 1])
