@@ -2521,6 +2521,28 @@ bool use_partial_query_tiles(int64_t seq_len, bool causal) {
     return seq_len < 1024 || (padded - seq_len) * 32 <= 3 * padded;
 }
 
+// Lengths that are not a multiple of 128: both kernels' times step up with every 256 workgroups,
+// one per CU, and a head's last 128-query group may be a quarter full, so the 128-query kernel
+// can be a step further up than its work is. Up to 128 keys (one group a head) it wins all the
+// same, with one step always, and from four on. Measured on MI355X (alternating runs, key-split 32
+// -> 128-query, us), by steps of the 32-query blocks and of the groups:
+//  - 4 and 2: 7.8 -> 8.3 (202 heads of N160), 9.1 -> 10.0 (112 of N288), 10.4 -> 11.7 (78 of
+//    N416), 17.4 -> 19.0 (35 of N928); 5 and 2: 10.5 -> 10.1 (114 of N288). The key-split kernel
+//    masks a last block of 16 keys and is slower there: 8.6 -> 9.1 (146 of N208), 12.0 -> 12.3 (68
+//    of N464), but 13.3 -> 13.3 (56 of N560) and 19.4 -> 18.6 (35 of N912).
+//  - 6 and 3: 10.7 -> 11.7 (300 of N160); 7 and 3: 14.4 -> 15.0 (189 of N288), 17.0 -> 18.1 (137
+//    of N416), and with 16 keys at the end 13.0 -> 11.7 (320 of N144); 8 and 3: 15.7 -> 15.1 (200
+//    of N288).
+bool key_split_has_fewer_rounds(int64_t batch_heads, int64_t seq_len) {
+    if (seq_len <= 128) return false;
+    const int64_t block_rounds = (batch_heads * ((seq_len + 31) / 32) + 255) / 256;
+    const int64_t group_rounds = (batch_heads * ((seq_len + 127) / 128) + 255) / 256;
+    const bool half_block = seq_len % 32 != 0;
+    if (group_rounds == 2) return block_rounds <= 4 && !(half_block && seq_len > 544);
+    if (group_rounds == 3) return block_rounds <= (half_block ? 6 : 7);
+    return false;
+}
+
 bool use_wide_kernel(int64_t batch_heads, int64_t seq_len, bool causal) {
     // Lengths that are a multiple of 128 and not of 256 keep the 128-query kernel.
     if (seq_len % 256 != 0 && (seq_len % 128 == 0 || !use_partial_query_tiles(seq_len, causal) || seq_len <= 128))
@@ -2554,7 +2576,8 @@ bool use_wide_kernel(int64_t batch_heads, int64_t seq_len, bool causal) {
 bool use_128_query_kernel(int64_t batch_heads, int64_t seq_len, bool causal) {
     if (seq_len % kQueryTileAlign != 0 && !use_partial_query_tiles(seq_len, causal)) return false;
     const int64_t blocks = batch_heads * ((seq_len + 31) / 32);  // four to a group
-    return blocks >= 4 * (causal ? 320 : 200);
+    return blocks >= 4 * (causal ? 320 : 200) &&
+           (seq_len % kQueryTileAlign == 0 || !key_split_has_fewer_rounds(batch_heads, seq_len));
 }
 
 // Causal problems of 320 to 512 groups of 128 queries (one round of the 128-query

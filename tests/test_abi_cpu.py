@@ -111,6 +111,22 @@ def test_forward_plan_follows_the_measured_thresholds(batch, heads, seq_len, cau
     assert capi.forward_plan(batch, heads, seq_len, causal) == kernel
 
 
+@pytest.mark.parametrize("heads, seq_len, split", [
+    # Two rounds of 128-query groups against four and five of 32-query blocks.
+    (202, 160, True), (204, 160, True), (205, 160, False), (113, 288, True), (114, 288, False), (37, 832, True),
+    (26, 1184, True), (146, 208, True), (147, 208, False), (200, 144, True), (205, 144, False),
+    (60, 528, True), (61, 528, False), (56, 560, False), (35, 912, False),
+    # Three rounds of groups.
+    (307, 160, True), (358, 160, True), (359, 160, False), (199, 288, True), (200, 288, False),
+    (307, 144, True), (308, 144, False),
+    # One round of groups, four, and lengths of one group.
+    (200, 112, False), (401, 48, False), (515, 64, False), (115, 208, False), (385, 160, False),
+])
+def test_ragged_lengths_take_the_kernel_of_fewer_rounds(heads, seq_len, split):
+    expected = K.FA2_KERNEL_KEY_SPLIT_32 if split else K.FA2_KERNEL_128_QUERY
+    assert capi.forward_plan(1, heads, seq_len, False) == expected
+
+
 @pytest.mark.parametrize("status, text", [
     (capi.FA2_STATUS_SUCCESS, "success"),
     (capi.FA2_STATUS_BAD_HEAD_DIM, "head dimension must equal 64"),
