@@ -75,16 +75,25 @@ hipError_t launch_copy(const void* src, void* dst, int64_t bytes, hipStream_t st
 //
 // kWide: head_dim a multiple of 4 and at most 2^16, and 16-byte aligned pointers: 16-byte
 // LDS-DMA, four rows an instruction. Otherwise 4-byte LDS-DMA, one row an instruction with a
-// descriptor of its own, for any head_dim and alignment.
+// descriptor of its own, for any head_dim and alignment. kNarrow (head_dim at most 16): rows of
+// 16 dimensions in LDS, four to a 4-byte LDS-DMA. The fetch instructions are what small
+// operands cost, so kNarrow and the one-row fetch of kSingle issue none for rows past seq_len,
+// whose products are not stored. FP32 VALU tile -> all 32 rows of a unit, one an instruction ->
+// this: B1 H8 N1024 D3 11.5 -> 11.9 -> 8.8 us, 2048 heads of N7 D3 6.8 -> 11.4 -> 5.2, of N7 D17
+// 11.5 -> 12.9 -> 7.9, 4096 heads of N1 D4 on 4-byte aligned storage 11.4 -> 20.6 -> 8.1.
 constexpr int kScoreTile = 64;
+constexpr int kNarrowDims = 16;
 
-template <bool kWide, bool kSingle>
+template <bool kWide, bool kSingle, bool kNarrow = false>
 __global__ __launch_bounds__(256) void scores_f32_kernel(const float* __restrict__ query,
                                                          const float* __restrict__ key,
                                                          float* __restrict__ scores, int seq_len,
                                                          int head_dim, uint32_t tiles, uint32_t ranges,
                                                          uint32_t total_blocks, float scale) {
-    constexpr int kUnitBytes = 32 * 256;
+    static_assert(!kNarrow || (kSingle && !kWide), "the narrow fetch");
+    constexpr int kPitch = kNarrow ? kNarrowDims * 4 : 256;  // bytes of a row in LDS
+    constexpr int kGroups = kPitch / 32;                      // of 8 dimensions
+    constexpr int kUnitBytes = 32 * kPitch;
     constexpr int kOutOfRange = 0x40000000;  // past every num_records here (a row of S is at most 2 MiB in HBM's 288 GB)
     constexpr int kParts = kSingle ? 2 : 1;  // waves that share the fetch of a unit
     constexpr int kSlotBytes = (kSingle ? 2 : 4) * kUnitBytes;  // K alone, or K and Q
@@ -117,20 +126,27 @@ __global__ __launch_bounds__(256) void scores_f32_kernel(const float* __restrict
         const int rows = min(32, seq_len - first);  // may be negative: nothing to fetch
         u32x4 d;
         d[3] = 0x00020000u;
-        if (kWide) {
+        if (kNarrow && rows <= 0) return;
+        if (kWide || kNarrow) {
             d[0] = __builtin_amdgcn_readfirstlane((uint32_t)base);
             d[1] = __builtin_amdgcn_readfirstlane((uint32_t)(base >> 32) & 0xffffu);
             d[2] = __builtin_amdgcn_readfirstlane(rows > 0 ? (uint32_t)(rows * row_bytes) - d0 * 4u : 0u);
 #pragma unroll
             for (int i = 0; i < 8 / kParts; ++i) {
                 const int n = i * kParts + part;
+                if (kNarrow && 4 * n >= rows) break;
                 const int row = 4 * n + (lane >> 4);
-                const int chunk16 = (lane & 15) ^ (row & 15);
-                const bool in = d0 + 4u * chunk16 < (uint32_t)head_dim;
-                dma16(d, lds + n * 1024, in ? (int)(row * row_bytes) + 16 * chunk16 : kOutOfRange);
+                if (kNarrow) {
+                    const int dim = (lane & 15) ^ ((n & 3) << 2);
+                    dma4(d, lds + n * 256, dim < head_dim ? (int)(row * row_bytes) + 4 * dim : kOutOfRange);
+                } else {
+                    const int chunk16 = (lane & 15) ^ (row & 15);
+                    const bool in = d0 + 4u * chunk16 < (uint32_t)head_dim;
+                    dma16(d, lds + n * 1024, in ? (int)(row * row_bytes) + 16 * chunk16 : kOutOfRange);
+                }
             }
         } else {
-            for (int row = part; row < 32; row += kParts) {
+            for (int row = part; row < (kSingle ? rows : 32); row += kParts) {
                 const uint64_t a = base + (uint64_t)row * row_bytes;
                 d[0] = __builtin_amdgcn_readfirstlane((uint32_t)a);
                 d[1] = __builtin_amdgcn_readfirstlane((uint32_t)(a >> 32) & 0xffffu);
@@ -151,7 +167,7 @@ __global__ __launch_bounds__(256) void scores_f32_kernel(const float* __restrict
     // waves read the one slot and refill the other.
     auto landed = [&]() { asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)\n\ts_barrier" ::: "memory"); };
 
-    const uint32_t lane_read = smem_addr + (uint32_t)(m * 256 + ((h ^ (m & 15)) << 4));
+    const uint32_t lane_read = smem_addr + (uint32_t)(m * kPitch + ((h ^ (kNarrow ? (m >> 2) & 3 : m & 15)) << 4));
     auto read = [&](int slot, int unit, int j) {
         return *reinterpret_cast<const FA2_LDS f32x4*>(
             (size_t)((lane_read ^ (uint32_t)(j << 5)) + (uint32_t)(slot * kSlotBytes + unit * kUnitBytes)));
@@ -163,11 +179,11 @@ __global__ __launch_bounds__(256) void scores_f32_kernel(const float* __restrict
         fetch(col_begin, 0, 0);
         landed();
 #pragma unroll
-        for (int j = 0; j < 8; ++j) qf[j] = read(1, wave >> 1, j);
+        for (int j = 0; j < kGroups; ++j) qf[j] = read(1, wave >> 1, j);
         // Every wave has read its Q before any wave's fetch refills slot 1. (The compiler may
         // sink LDS reads past a plain barrier; the asm takes their results.)
 #pragma unroll
-        for (int j = 0; j < 8; ++j) asm volatile("" : "+v"(qf[j]));
+        for (int j = 0; j < kGroups; ++j) asm volatile("" : "+v"(qf[j]));
         asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
     } else {
         fetch(col_begin, 0, 0);
@@ -198,7 +214,7 @@ __global__ __launch_bounds__(256) void scores_f32_kernel(const float* __restrict
             if (chunk + 1 < chunks) fetch(col, chunk + 1, slot ^ 1);
             else if (col + 1 < col_end) fetch(col + 1, 0, slot ^ 1);
             const int groups = (int)min(8u, ((uint32_t)head_dim - (uint32_t)chunk * 64u + 7u) / 8u);  // of 8 dimensions
-            if (groups == 8) {
+            if (!kNarrow && groups == 8) {
                 f32x4 kf[8];
 #pragma unroll
                 for (int j = 0; j < 8; ++j) kf[j] = read(slot, wave & 1, j);
@@ -207,7 +223,7 @@ __global__ __launch_bounds__(256) void scores_f32_kernel(const float* __restrict
                 for (int j = 0; j < 8; ++j) multiply(kSingle ? qf[j] : read(slot, 2 + (wave >> 1), j), kf[j]);
             } else {
 #pragma unroll
-                for (int j = 0; j < 7; ++j)
+                for (int j = 0; j < min(7, kGroups); ++j)
                     if (j < groups) multiply(kSingle ? qf[j] : read(slot, 2 + (wave >> 1), j), read(slot, wave & 1, j));
             }
             if (chunk + 1 < chunks) landed();
@@ -222,7 +238,7 @@ __global__ __launch_bounds__(256) void scores_f32_kernel(const float* __restrict
         for (int i = 0; i < 16; ++i)
             __builtin_amdgcn_raw_buffer_store_b32(__float_as_uint((acc[0][i] + acc[1][i]) * scale), out,
                                                   lane_offset + (8 * (i >> 2) + (i & 3)) * seq_len * 4, 0, 0);
-        asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
+        if (col + 1 < col_end) asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
     }
 }
 
@@ -301,8 +317,11 @@ extern "C" int fa2_attention_scores_f32(const float* query, const float* key, fl
     const int64_t x = total < kMaxX ? total : kMaxX;
     const dim3 grid((unsigned)x, (unsigned)((total + x - 1) / x));
     const bool wide = head_dim % 4 == 0 && head_dim <= 65536 && aligned_to(query, 16) && aligned_to(key, 16);
-    const auto kernel = head_dim <= 64 ? (wide ? scores_f32_kernel<true, true> : scores_f32_kernel<false, true>)
-                                       : (wide ? scores_f32_kernel<true, false> : scores_f32_kernel<false, false>);
+    // Up to 16 keys the narrow fetch also beats the wide one (2048 heads of D8 at N7 6.5 -> 5.1 us,
+    // at N16 6.5 -> 5.6), beyond no longer (B1 H8 N1024 D8 8.5 -> 8.6).
+    const auto kernel = head_dim <= kNarrowDims && (!wide || seq_len <= 16) ? scores_f32_kernel<false, true, true>
+                        : head_dim <= 64 ? (wide ? scores_f32_kernel<true, true> : scores_f32_kernel<false, true>)
+                                         : (wide ? scores_f32_kernel<true, false> : scores_f32_kernel<false, false>);
     hipLaunchKernelGGL(kernel, grid, dim3(256), 0, static_cast<hipStream_t>(stream), query, key, scores, (int)seq_len,
                        (int)head_dim, (uint32_t)tiles, (uint32_t)ranges, (uint32_t)total, scale);
     return hip_status(hipGetLastError());

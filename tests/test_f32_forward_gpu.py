@@ -169,6 +169,22 @@ def test_scores_edges(seq_len, dim, offset):
     assert ((out - expected).abs() <= bound).all()
 
 
+# The narrow fetch: up to 16 dimensions, four rows an instruction; its edges in dimensions and rows,
+# from one block to ranges of several, beside the fetches that take over above 16 dimensions and,
+# for 16-byte aligned rows of whole chunks, above 16 rows.
+@pytest.mark.parametrize("offset", [0, 1])
+@pytest.mark.parametrize("batch_heads, seq_len", [(3, 1), (2, 4), (2, 5), (2, 16), (2, 17), (2, 62), (2, 97), (70, 300)])
+@pytest.mark.parametrize("dim", [1, 2, 5, 8, 9, 15, 16, 17])
+def test_scores_narrow_fetch(batch_heads, seq_len, dim, offset):
+    q, k, _ = _inputs(batch_heads, seq_len, dim, seed=dim, offset=offset)
+    print(batch_heads, seq_len, dim, offset, flush=True)
+    out = capi.attention_scores_f32(q, k).double().cpu()
+    exact_q, exact_k = q.double().cpu(), k.double().cpu()
+    expected = exact_q @ exact_k.transpose(-1, -2) / math.sqrt(dim)
+    bound = (dim / 2 + 3) * 2.0 ** -24 * (exact_q.abs() @ exact_k.abs().transpose(-1, -2)) / math.sqrt(dim)
+    assert ((out - expected).abs() <= bound).all()
+
+
 def test_scores_nan_and_infinity():
     q, k, _ = _inputs(2, 70, 64, seed=5)
     q[0, 0, 3, 5], q[0, 1, 65, 63], k[0, 0, 40, 2], k[0, 1, 1, 0] = math.nan, math.inf, -math.inf, math.inf

@@ -104,7 +104,7 @@ def test_scores_barriers_wait_for_lds_reads(kernels):
     """Behind each barrier of the scores kernel another wave's LDS-DMA refills the ring slot that
     this wave read before it, so the wave waits for its reads at the barrier itself."""
     scores = {name: body for name, body in kernels.items() if "scores_f32_kernel" in name}
-    assert len(scores) == 4
+    assert scores
     for name, body in scores.items():
         barriers = [at for at, instruction in enumerate(body) if instruction == "s_barrier"]
         assert barriers
