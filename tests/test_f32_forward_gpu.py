@@ -178,6 +178,33 @@ def test_scores_edges(seq_len, dim, offset):
     assert ((out - expected).abs() <= bound).all()
 
 
+def _blocks_and_ranges(batch_heads, seq_len):
+    """64-column blocks of a row of blocks, and the workgroups they are dealt to: four workgroups
+    per CU in all, and at most eight blocks each."""
+    blocks = -(-seq_len // 64)
+    return blocks, min(blocks, max(-(-blocks // 8), -(-1024 // (batch_heads * blocks))))
+
+
+# Workgroups of several blocks: the next block's operands land in the other ring slot while a
+# block is multiplied and stored. Two blocks each, one or two, five, six or seven, and eight; one,
+# two, three and four chunks of dimensions a block.
+@pytest.mark.parametrize("offset", [0, 1])
+@pytest.mark.parametrize("batch_heads, seq_len", [(8, 1024), (8, 1000), (40, 333), (64, 600), (20, 2100), (128, 512)])
+@pytest.mark.parametrize("dim", [3, 60, 64, 68, 130, 200])
+def test_scores_of_several_blocks(batch_heads, seq_len, dim, offset):
+    blocks, ranges = _blocks_and_ranges(batch_heads, seq_len)
+    assert ranges < blocks
+    q, k, _ = _inputs(batch_heads, seq_len, dim, seed=dim, offset=offset)
+    print(batch_heads, seq_len, dim, offset, flush=True)
+    out = capi.attention_scores_f32(q, k)
+    for head in range(batch_heads):
+        # On the GPU: FP64 products of a plain matrix and a transposed copy.
+        exact_q, exact_k = q[0, head].double(), k[0, head].double().t().contiguous()
+        expected = exact_q @ exact_k / math.sqrt(dim)
+        bound = (dim / 2 + 3) * 2.0 ** -24 * (exact_q.abs() @ exact_k.abs()) / math.sqrt(dim)
+        assert ((out[0, head].double() - expected).abs() <= bound).all()
+
+
 # The narrow fetch: up to 16 dimensions, four rows an instruction; its edges in dimensions and rows,
 # from one block to ranges of several, beside the fetches that take over above 16 dimensions and,
 # for 16-byte aligned rows of whole chunks, above 16 rows.
