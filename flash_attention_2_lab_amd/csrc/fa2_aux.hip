@@ -77,12 +77,16 @@ hipError_t launch_copy(const void* src, void* dst, int64_t bytes, hipStream_t st
 // LDS-DMA, four rows an instruction. Otherwise 4-byte LDS-DMA, one row an instruction with a
 // descriptor of its own, for any head_dim and alignment. kNarrow (head_dim at most 16): rows of
 // 16 dimensions in LDS, four to a 4-byte LDS-DMA. The fetch instructions are what small
-// operands cost, so kNarrow and the one-row fetch of kSingle issue none for rows past seq_len,
-// whose products are not stored. FP32 VALU tile -> all 32 rows of a unit, one an instruction ->
-// this: B1 H8 N1024 D3 11.5 -> 11.9 -> 8.8 us, 2048 heads of N7 D3 6.8 -> 11.4 -> 5.2, of N7 D17
-// 11.5 -> 12.9 -> 7.9, 4096 heads of N1 D4 on 4-byte aligned storage 11.4 -> 20.6 -> 8.1.
+// operands cost, so kNarrow, the one-row fetch of kSingle and any one-row fetch of a unit of up to
+// kFewRows rows issue none for rows past seq_len, whose products are not stored. FP32 VALU tile ->
+// all 32 rows of a unit, one an instruction -> this: B1 H8 N1024 D3 11.5 -> 11.9 -> 8.8 us, 2048
+// heads of N7 D3 6.8 -> 11.4 -> 5.2, of N7 D17 11.5 -> 12.9 -> 7.9, 4096 heads of N1 D4 on 4-byte
+// aligned storage 11.4 -> 20.6 -> 8.1, of N1 D65 47.2 -> 52.3 -> 33.4, 2048 of N16 D65 26.4 -> 27.5 ->
+// 22.4. Past 64 dimensions a loop to the last row alone lost at 32 rows (8 heads of N1000 D65 33.7
+// -> 28.6 -> 30.7, with this rule 29.0) and at 48 keys (700 heads 15.1 -> 12.6 -> 13.9, with it 12.4).
 constexpr int kScoreTile = 64;
 constexpr int kNarrowDims = 16;
+constexpr int kFewRows = 24;
 
 template <bool kWide, bool kSingle, bool kNarrow = false>
 __global__ __launch_bounds__(256) void scores_f32_kernel(const float* __restrict__ query,
@@ -146,12 +150,17 @@ __global__ __launch_bounds__(256) void scores_f32_kernel(const float* __restrict
                 }
             }
         } else {
-            for (int row = part; row < (kSingle ? rows : 32); row += kParts) {
+            auto fetch_row = [&](int row, bool exists) {
                 const uint64_t a = base + (uint64_t)row * row_bytes;
                 d[0] = __builtin_amdgcn_readfirstlane((uint32_t)a);
                 d[1] = __builtin_amdgcn_readfirstlane((uint32_t)(a >> 32) & 0xffffu);
-                d[2] = __builtin_amdgcn_readfirstlane(row < rows ? min(64u, (uint32_t)head_dim - d0) * 4u : 0u);
+                d[2] = __builtin_amdgcn_readfirstlane(exists ? min(64u, (uint32_t)head_dim - d0) * 4u : 0u);
                 dma4(d, lds + row * 256, (lane << 2) ^ ((row & 15) << 4));
+            };
+            if (kSingle || rows <= kFewRows) {
+                for (int row = part; row < rows; row += kParts) fetch_row(row, true);
+            } else {
+                for (int row = 0; row < 32; ++row) fetch_row(row, row < rows);
             }
         }
     };

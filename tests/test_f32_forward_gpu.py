@@ -221,6 +221,19 @@ def test_scores_narrow_fetch(batch_heads, seq_len, dim, offset):
     assert ((out - expected).abs() <= bound).all()
 
 
+# The one-row fetch past 64 dimensions stops at the last row of units of up to 24 rows and fetches 32
+# of larger ones; lengths on both sides, in the first and in the second unit of a block.
+@pytest.mark.parametrize("batch_heads, seq_len", [(3, 1), (2, 24), (2, 25), (2, 32), (2, 56), (2, 57), (2, 88), (40, 345)])
+@pytest.mark.parametrize("dim", [65, 129])
+def test_scores_few_rows(batch_heads, seq_len, dim):
+    q, k, _ = _inputs(batch_heads, seq_len, dim, seed=dim, offset=1)
+    out = capi.attention_scores_f32(q, k).double().cpu()
+    exact_q, exact_k = q.double().cpu(), k.double().cpu()
+    expected = exact_q @ exact_k.transpose(-1, -2) / math.sqrt(dim)
+    bound = (dim / 2 + 3) * 2.0 ** -24 * (exact_q.abs() @ exact_k.abs().transpose(-1, -2)) / math.sqrt(dim)
+    assert ((out - expected).abs() <= bound).all()
+
+
 def test_scores_nan_and_infinity():
     q, k, _ = _inputs(2, 70, 64, seed=5)
     q[0, 0, 3, 5], q[0, 1, 65, 63], k[0, 0, 40, 2], k[0, 1, 1, 0] = math.nan, math.inf, -math.inf, math.inf
