@@ -2510,15 +2510,11 @@ double modeled_rounds(int64_t workgroups, double lone_round) {
 // from 48 on the same crossover as at whole tiles holds when work is counted in 32-query
 // blocks. Measured on MI355X (graph replays, key-split 32 -> 128- or 256-query): B4 H16
 // N2032 134 -> 73 us, B16 H16 N4080 1805 -> 1032 us, B1 H25 N1008 19.0 -> 13.9 us, 512 heads
-// of N240 31 -> 19.5 us, of N144 (44% padding) 19.2 -> 12.9 us, 256 heads of N48 (below the
-// crossover) 4.1 -> 4.1 us.
-// From 1024 on, lengths whose 128-query tiles are more than 3/32 padding (N = 1040 alone)
-// stay on the key-split kernel, which fa2_forward_plan has always named for them, at a cost:
-// 43 against 34 us at 64 heads.
+// of N240 31 -> 19.5 us, of N144 (44% padding) 19.2 -> 12.9 us, 25, 64 and 512 of
+// N1040 (10%) 19.7 -> 14.7, 40.8 -> 33.1 and 303 -> 177 us, 256 heads of N48 (below the crossover)
+// 4.1 -> 4.1 us.
 bool use_partial_query_tiles(int64_t seq_len, bool causal) {
-    if (causal || seq_len <= 32) return false;
-    const int64_t padded = (seq_len + 127) / 128 * 128;
-    return seq_len < 1024 || (padded - seq_len) * 32 <= 3 * padded;
+    return !causal && seq_len > 32;
 }
 
 // Lengths that are not a multiple of 128: both kernels' times step up with every 256 workgroups,

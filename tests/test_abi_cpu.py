@@ -95,8 +95,9 @@ K = capi
     (1, 4, 1040, False, K.FA2_KERNEL_KEY_SPLIT_64_DMA_WAVES), (1, 2, 2000, False, K.FA2_KERNEL_KEY_SPLIT_64_DMA_WAVES),
     (1, 1, 2064, False, K.FA2_KERNEL_KEY_SPLIT_8_WAVES),
     # Sequence lengths the production entry rejects but the Bc16/Bc32 entries take
-    # (partial last block) run the key-split kernel.
-    (4, 64, 1040, False, K.FA2_KERNEL_KEY_SPLIT_32), (1, 2, 80, False, K.FA2_KERNEL_KEY_SPLIT_32), (1, 2, 240, False, K.FA2_KERNEL_KEY_SPLIT_64),
+    # (partial last block) run the key-split kernel while small, then the 128- and 256-query ones.
+    (4, 64, 1040, False, K.FA2_KERNEL_128_QUERY), (5, 60, 1040, False, K.FA2_KERNEL_256_QUERY),
+    (1, 24, 1040, False, K.FA2_KERNEL_KEY_SPLIT_32), (1, 25, 1040, False, K.FA2_KERNEL_128_QUERY), (1, 2, 80, False, K.FA2_KERNEL_KEY_SPLIT_32), (1, 2, 240, False, K.FA2_KERNEL_KEY_SPLIT_64),
     # Causal 256-query: pairs of tiles at T = 2, 4 and 8, head groups
     # at T >= 16 or odd; split pairs from 4096 keys at 320-512 groups of 128.
     (32, 16, 1024, True, K.FA2_KERNEL_256_QUERY_PAIRS), (8, 16, 2048, True, K.FA2_KERNEL_256_QUERY_PAIRS),

@@ -17,7 +17,7 @@ K128, K256 = capi.FA2_KERNEL_128_QUERY, capi.FA2_KERNEL_256_QUERY
 CASES = [
     (401, 48, K128), (267, 80, K128), (201, 112, K128), (512, 144, K256), (1000, 176, K256),
     (300, 272, K128), (512, 208, K256), (64, 528, K128), (256, 496, K256), (25, 1008, K128),
-    (14, 2064, K128), (64, 2032, K256), (256, 1008, K256), (100, 2320, K256),
+    (14, 2064, K128), (64, 2032, K256), (256, 1008, K256), (100, 2320, K256), (64, 1040, K128), (300, 1040, K256),
 ]
 
 
