@@ -66,8 +66,8 @@ hipError_t launch_copy(const void* src, void* dst, int64_t bytes, hipStream_t st
 // B1 H8 N1024): a step (one chunk of one block) fetches the next step's operands before its
 // products, and the stores of a block run beside the products of the next. kSingle
 // (head_dim <= 64) keeps Q in registers, so that a step fetches K alone and 32 KiB of LDS
-// leave room for five workgroups per CU. A register of the accumulator is stored as two
-// 128-byte row segments; rows and columns past seq_len fall outside num_records.
+// are enough; 112 VGPRs leave room for four workgroups per CU. A register of the accumulator is
+// stored as two 128-byte row segments; rows and columns past seq_len fall outside num_records.
 // Measured on MI355X (graph replays, FP32 VALU tile with 4-byte LDS reads -> this): B1 H8
 // N1024 D64 31.5 -> 15.6 us, D16 12.4 -> 9.4 us; B1 H8 N2048 D64 95 -> 47 us; B4 H8 N2048
 // D128 634 -> 348 us; B1 H1 N64 D64 9.6 -> 3.3 us. One block per workgroup, its phases in

@@ -46,7 +46,6 @@ def _exact(q, k, v):
     (130, 40), (257, 1), (260, 31), (129, 64), (65, 129), (52, 161), (9, 1025)])
 def test_f32_forward_edges(batch_heads, seq_len, dim, offset):
     q, k, v = _inputs(batch_heads, seq_len, dim, offset=offset)
-    print(batch_heads, seq_len, dim, offset, flush=True)
     out = capi.attention_forward_f32(q, k, v).double().cpu()
     expected = _exact(q, k, v)
     torch.testing.assert_close(out, expected, atol=ATOL, rtol=0)
@@ -169,7 +168,6 @@ def test_f32_forward_keeps_small_weights(batch_heads, case):
 @pytest.mark.parametrize("dim", [1, 3, 4, 60, 64, 68, 130, 256])
 def test_scores_edges(seq_len, dim, offset):
     q, k, _ = _inputs(3, seq_len, dim, seed=dim, offset=offset)
-    print(seq_len, dim, offset, flush=True)
     out = capi.attention_scores_f32(q, k).double().cpu()
     exact_q, exact_k = q.double().cpu(), k.double().cpu()
     expected = exact_q @ exact_k.transpose(-1, -2) / math.sqrt(dim)
@@ -195,7 +193,6 @@ def test_scores_of_several_blocks(batch_heads, seq_len, dim, offset):
     blocks, ranges = _blocks_and_ranges(batch_heads, seq_len)
     assert ranges < blocks
     q, k, _ = _inputs(batch_heads, seq_len, dim, seed=dim, offset=offset)
-    print(batch_heads, seq_len, dim, offset, flush=True)
     out = capi.attention_scores_f32(q, k)
     for head in range(batch_heads):
         # On the GPU: FP64 products of a plain matrix and a transposed copy.
@@ -213,7 +210,6 @@ def test_scores_of_several_blocks(batch_heads, seq_len, dim, offset):
 @pytest.mark.parametrize("dim", [1, 2, 5, 8, 9, 15, 16, 17])
 def test_scores_narrow_fetch(batch_heads, seq_len, dim, offset):
     q, k, _ = _inputs(batch_heads, seq_len, dim, seed=dim, offset=offset)
-    print(batch_heads, seq_len, dim, offset, flush=True)
     out = capi.attention_scores_f32(q, k).double().cpu()
     exact_q, exact_k = q.double().cpu(), k.double().cpu()
     expected = exact_q @ exact_k.transpose(-1, -2) / math.sqrt(dim)

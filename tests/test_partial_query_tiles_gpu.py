@@ -40,7 +40,6 @@ def _run(q, k, v):
 
 @pytest.mark.parametrize("heads, seq_len, kernel", CASES)
 def test_partial_query_tiles_match_oracle(heads, seq_len, kernel):
-    print(heads, seq_len, kernel, flush=True)
     assert capi.forward_plan(1, heads, seq_len, False) == kernel
     q, k, v = _inputs(heads, seq_len, seed=seq_len)
     # Growing key norms make later tiles, the partial one among them, move the running max.
