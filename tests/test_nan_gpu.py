@@ -22,7 +22,8 @@ Infinities are honoured (no -fno-honor-infs) and follow the formula the same way
   rows) and -inf in the rows whose q[e] < 0 (key j gets probability 0, the row stays
   finite);
 * +inf in value (j, d) makes dimension d infinite in every row that sees key j, with
-  the same exception as the NaN case for causal rows i < j.
+  the same exception as the NaN case for causal rows i < j;
+* -inf scores over whole key tiles, from a row's first on, leave the later keys' average.
 """
 
 from __future__ import annotations
@@ -161,6 +162,25 @@ def test_inf_in_key_row(shape, causal, kernel):
         nan_rows[:j] = False
     assert torch.equal(torch.isnan(expected[b, h]).all(-1), nan_rows)
     assert 0 < int(nan_rows.sum()) < n - j
+    _check_nonfinite(ENTRY(q.cuda(), k.cuda(), v.cuda(), causal), expected)
+
+
+# Ragged lengths on the 128- and 256-query kernels, beside the shapes above.
+HIDDEN = SHAPES + [((1, 25, 1008), False, capi.FA2_KERNEL_128_QUERY), ((4, 64, 2032), False, capi.FA2_KERNEL_256_QUERY)]
+
+
+@pytest.mark.parametrize("shape, causal, kernel", HIDDEN, ids=[f"{'causal' if c else 'noncausal'}-{s}" for s, c, _ in HIDDEN])
+def test_inf_hides_leading_keys(shape, causal, kernel):
+    """Scores of -inf over whole key tiles from the first on: the later keys' average."""
+    assert capi.forward_plan(*shape, causal) == kernel
+    q, k, v = _inputs(shape, seed=77)
+    n = shape[2]
+    b, h, hidden = shape[0] - 1, shape[1] - 1, min(n // 2, 320)
+    q[b, h, :, 0] = q[b, h, :, 0].abs() + 0.25
+    k[b, h, :hidden, 0] = float("-inf")
+    expected = attention_reference_fp32(q, k, v, causal=causal)
+    # Causal rows that see hidden keys only are NaN.
+    assert int(torch.isnan(expected).sum()) == (64 * hidden if causal else 0)
     _check_nonfinite(ENTRY(q.cuda(), k.cuda(), v.cuda(), causal), expected)
 
 
